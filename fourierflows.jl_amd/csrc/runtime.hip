@@ -87,7 +87,11 @@ int dev_alloc(void** p, size_t bytes) {
     return fail(e == hipErrorOutOfMemory ? FFHIP_ERR_OOM : FFHIP_ERR_HIP, "hipMalloc(%zu) failed: %s", bytes,
                 hipGetErrorString(e));
   }
+  // The fill runs on the null stream and may still be under way when hipMemset
+  // returns; a stream made non-blocking does not wait for it, so the caller's
+  // first kernel could write the array before the zeros arrive.
   e = hipMemset(*p, 0, bytes);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   if (e != hipSuccess) {
     (void)hipFree(*p);
     *p = nullptr;

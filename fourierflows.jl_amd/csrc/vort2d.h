@@ -209,6 +209,8 @@ int vort_export(int prec, const VortGeom& g, void* sol, const void* U, const dou
                 int64_t nsteps, hipStream_t st);
 // true when the row kernel takes this geometry
 bool vort_row_ok(int prec, const VortGeom& g);
+// true while st is being captured: it takes plain launches only, no allocation and no graph
+bool vort_capturing(hipStream_t st);
 int vort_col_explicit(int prec, const VortGeom& g, const VortColArgs& a, hipStream_t st);
 // one row pass / column stage (0..4, kVExplicit) of a state, on the kernels its axes take
 int vort_row_any(int prec, const VortState* s, const VortRowArgs& a, hipStream_t st);

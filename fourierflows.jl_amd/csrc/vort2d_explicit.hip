@@ -207,6 +207,8 @@ int fused_explicit_run(ffhip_op* op, ffhip_rk4* ts, int kind, void* sol, double 
   VortState* s = ts->cplx_coef ? nullptr : vort_state(op, st);
   if (!s || (!s->mixx && !vort_row_ok(op->prec, s->g))) return FFHIP_OK;
   const size_t bytes = (size_t)s->g.TX * s->g.KY * kVCB * sizeof(double);
+  // a capture cannot allocate: the plan-based path takes its first run
+  if ((!s->XL || (ts->filter && !s->XF)) && vort_capturing(st)) return FFHIP_OK;
   if ((!s->XL && dev_alloc(&s->XL, bytes) != FFHIP_OK) ||
       (ts->filter && !s->XF && dev_alloc(&s->XF, bytes) != FFHIP_OK)) {
     clear_error();  // no room for the blocked copies: the plan-based path runs

@@ -487,8 +487,7 @@ void fused_destroy(ffhip_op* op) {
   op->fused = op->mixed = nullptr;
 }
 
-// a stream under capture takes plain launches only: no allocation, no graph
-static bool capturing(hipStream_t st) {
+bool vort_capturing(hipStream_t st) {
   hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &c) != hipSuccess) {
     (void)hipGetLastError();
@@ -504,7 +503,7 @@ static bool capturing(hipStream_t st) {
 VortState* vort_state(ffhip_op* op, hipStream_t st) {
   if (op->kind != FFHIP_OP_VORTICITY2D) return nullptr;
   if (op->fused) return reinterpret_cast<VortState*>(op->fused);
-  if (op->mixed || op->no_mixed || capturing(st)) return reinterpret_cast<VortState*>(op->mixed);
+  if (op->mixed || op->no_mixed || vort_capturing(st)) return reinterpret_cast<VortState*>(op->mixed);
   op->no_mixed = true;
   VortState s;
   const int64_t nx = op->n[0], ny = op->n[1];
@@ -614,7 +613,7 @@ static int vrun(ffhip_op* op, VortState* s, ffhip_etdrk4* ts, void* sol, int64_t
   // set outside the capture); later runs find it ready.  The last step runs
   // eagerly because it differs.  Profiled runs stay eager: they time each
   // launch; so do runs that a caller captures.
-  const bool graphs = !g_prof_on && vort_graphs_on() && !capturing(st);
+  const bool graphs = !g_prof_on && vort_graphs_on() && !vort_capturing(st);
   if (graphs && left >= 1 && (!s->exec || s->graph_packed != ts->packed || s->graph_filter != (ts->filter != nullptr))) {
     FF_TRY(step(st, left == 1));
     --left;
