@@ -26,6 +26,7 @@ struct ffhip_op {
   void* mixed = nullptr;   // the same on other grids (mixed-radix passes), made at the first run
   bool no_mixed = false;   // that state is not wanted, not possible or found no memory
   bool no_modes = false;   // tracer: transforms also where the mode stencil would do
+  void* flags = nullptr;   // tracer: three ints of the mode stencil (tracer_modes.hip)
   void* fused3 = nullptr;  // fused RK4 state of the tracer (power-of-two 3D grids)
 };
 

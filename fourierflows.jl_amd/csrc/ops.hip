@@ -511,6 +511,7 @@ static void op_free(ffhip_op* op) {
   for (auto& p : op->spec) dev_free(p);
   for (auto& p : op->phys) dev_free(p);
   dev_free(op->tables);
+  dev_free(op->flags);
   delete op;
 }
 
@@ -591,7 +592,8 @@ int ffhip_op_create(ffhip_op** out, int kind, int prec, int ndim, const int64_t*
       }
       off += 2 * ns[d];
     }
-    rc = dev_alloc(&op->tables, tab.size() * sizeof(double));
+    rc = dev_alloc(&op->flags, 3 * sizeof(int));
+    if (rc == FFHIP_OK) rc = dev_alloc(&op->tables, tab.size() * sizeof(double));
     if (rc == FFHIP_OK) {
       hipError_t e = hipMemcpy(op->tables, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice);
       if (e != hipSuccess) rc = fail(FFHIP_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));

@@ -12,6 +12,10 @@
 // of the kx = 0 plane that is not Hermitian, which also supplies the modes of
 // negative kx.
 //
+// A mode that is infinite or NaN makes every grid value NaN and with them N on
+// the whole kept band.  The stencil alone would hand it to the neighbours only,
+// so the passes note one they read, and the last launch fills the band.
+//
 // An RK4 stage is one kernel over the kept band: it reads the stage state with
 // its neighbours (from cache), the state and L, and writes RHS and the next
 // stage state, so memory bounds it: 256^3 FP32 (2.5 M kept modes) moves about
@@ -50,6 +54,8 @@ struct TmArgs {
   const double* L;
   const double* F;  // filter or null
   double h, h6;
+  int* bad;   // a mode that is not finite: [0] in the run, [1] in stage 1's state, [2] in calcN's
+  int first;  // stage 1 of a run
 };
 
 // a field of modes by signed wavenumbers: rows of ny_, planes of nz_ (native: ny, nz; packed: KY, KZ)
@@ -71,7 +77,7 @@ struct TmField {
     cplx<R> a = neg ? get(g, -kx, -l, -m) : get(g, kx, l, m);
     if (kx == 0) {
       const cplx<R> b = get(g, 0, -l, -m);
-      a = mkc<R>(R(0.5) * (a.x + b.x), R(0.5) * (a.y - b.y));
+      a = mkc<R>(R(0.5) * (a.x + b.x), l == 0 && m == 0 ? R(0) : R(0.5) * (a.y - b.y));  // the mean is real
     }
     return neg ? cconj<R>(a) : a;
   }
@@ -112,7 +118,9 @@ template <typename R, int STAGE, bool SLOW>
 __device__ __forceinline__ void tm_read(const TmGeom& g, const TmArgs& a, const TmField<R>& f, int kx, int l, int m,
                                         TmVal<R>& v) {
   v.n = tm_N<R, SLOW>(g, f, kx, l, m);
-  if constexpr (STAGE > 0) {
+  if constexpr (STAGE == 0) {
+    v.x = f.p[f.at(kx, l, m)];
+  } else {
     const uint32_t nat = TmField<R>{nullptr, g.nkr, g.ny, g.nz}.at(kx, l, m);
     v.u = reinterpret_cast<const cplx<R>*>(a.sol)[nat];
     v.x = STAGE == 1 ? v.u : f.p[f.at(kx, l, m)];
@@ -147,11 +155,18 @@ __device__ __forceinline__ void tm_write(const TmGeom& g, const TmArgs& a, int k
     }
   }
 }
+// 0 where z is finite, else NaN
+template <typename R>
+__device__ __forceinline__ R tm_nan(cplx<R> z) {
+  return z.x * R(0) + z.y * R(0);
+}
+// one mode; a mode that is not finite is noted, but for the imaginary part of the mean, which c2r ignores
 template <typename R, int STAGE, bool SLOW>
-__device__ __forceinline__ void tm_mode(const TmGeom& g, const TmArgs& a, const TmField<R>& f, int kx, int l, int m) {
+__device__ __forceinline__ R tm_mode(const TmGeom& g, const TmArgs& a, const TmField<R>& f, int kx, int l, int m) {
   TmVal<R> v;
   tm_read<R, STAGE, SLOW>(g, a, f, kx, l, m, v);
   tm_write<R, STAGE>(g, a, kx, l, m, v);
+  return tm_nan<R>(SLOW && kx == 0 && l == 0 && m == 0 ? mkc<R>(v.x.x, 0) : v.x);
 }
 
 // Workgroups: groups of kTmPlanes consecutive m in order, each first the
@@ -162,6 +177,14 @@ __device__ __forceinline__ void tm_mode(const TmGeom& g, const TmArgs& a, const 
 // takes a contiguous range of m: neighbouring planes are read from its L2.
 template <typename R, int STAGE>
 __global__ void __launch_bounds__(kTmThreads) k_tracer_modes(TmGeom g, TmArgs a) {
+  // bad[0] of a run: cleared in its first stage 1, whose finds go to bad[1];
+  // stage 2 takes those over and stage 3 clears bad[1], so no launch sets a
+  // flag that it clears or reads
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (STAGE == 1 && a.first) a.bad[0] = 0;
+    if (STAGE == 2 && a.bad[1]) a.bad[0] = 1;
+    if (STAGE == 3) a.bad[1] = 0;
+  }
   const int blk = (int)(blockIdx.x % 8) * g.per_xcd + (int)(blockIdx.x / 8);
   if (blk >= g.nblk) return;
   const int tiles = g.tfast + g.tslow;
@@ -185,17 +208,22 @@ __global__ void __launch_bounds__(kTmThreads) k_tracer_modes(TmGeom g, TmArgs a)
   const TmField<R> f{reinterpret_cast<const cplx<R>*>(a.x), native ? g.nkr : g.KX, native ? g.ny : g.KY,
                      native ? g.nz : g.KZ};
   const int m0 = g.mmin + mg * kTmPlanes, m1 = min(m0 + kTmPlanes - 1, g.mmax);
+  R nan = 0;  // stays 0 while every mode is finite
   if (slow) {
-    if (m0 + j <= m1) tm_mode<R, STAGE, true>(g, a, f, kx, l, m0 + j);
+    if (m0 + j <= m1) nan = tm_mode<R, STAGE, true>(g, a, f, kx, l, m0 + j);
   } else if (m1 - m0 == kTmPlanes - 1) {
     TmVal<R> v[kTmPlanes];  // all reads before the first store, so that they are in flight together
 #pragma unroll
     for (int j = 0; j < kTmPlanes; ++j) tm_read<R, STAGE, false>(g, a, f, kx, l, m0 + j, v[j]);
 #pragma unroll
-    for (int j = 0; j < kTmPlanes; ++j) tm_write<R, STAGE>(g, a, kx, l, m0 + j, v[j]);
+    for (int j = 0; j < kTmPlanes; ++j) {
+      tm_write<R, STAGE>(g, a, kx, l, m0 + j, v[j]);
+      nan += tm_nan<R>(v[j].x);
+    }
   } else {
-    for (int m = m0; m <= m1; ++m) tm_mode<R, STAGE, false>(g, a, f, kx, l, m);
+    for (int m = m0; m <= m1; ++m) nan += tm_mode<R, STAGE, false>(g, a, f, kx, l, m);
   }
+  if (nan != R(0)) a.bad[STAGE == 0 ? 2 : STAGE == 1] = 1;
 }
 
 __device__ __forceinline__ bool tm_kept(const TmGeom& g, int64_t idx) {
@@ -205,23 +233,36 @@ __device__ __forceinline__ bool tm_kept(const TmGeom& g, int64_t idx) {
   return ix < g.KX && (iy <= g.lmax || iy >= g.ny + g.lmin) && (iz <= g.mmax || iz >= g.nz + g.mmin);
 }
 
-// modes outside the kept band: N = 0
+static __global__ void k_tracer_clear(int* bad) { bad[2] = 0; }
+
+// modes outside the kept band: N = 0; on the band NaN if a mode was not finite
 template <typename R>
-__global__ void __launch_bounds__(kTmThreads) k_tracer_outside_zero(cplx<R>* N, int64_t total, TmGeom g) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x)
-    if (!tm_kept(g, i)) N[i] = mkc<R>(0, 0);
+__global__ void __launch_bounds__(kTmThreads) k_tracer_outside_zero(cplx<R>* N, int64_t total, const int* bad,
+                                                                    TmGeom g) {
+  const bool fill = bad[2] != 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    if (!tm_kept(g, i))
+      N[i] = mkc<R>(0, 0);
+    else if (fill)
+      N[i] = mkc<R>((R)NAN, (R)NAN);
+  }
 }
 
-// and the RK4 steps of du/dt = L u there, with the stages' roundings
+// The same after a run: outside the band the RK4 steps of du/dt = L u, with the
+// stages' roundings (a zero stays one where L and the filter are finite)
 template <typename R>
 __global__ void __launch_bounds__(kTmThreads) k_tracer_outside(cplx<R>* sol, const double* L, const double* F,
                                                                double h2, double h, double h6, int64_t nsteps,
-                                                               int64_t total, TmGeom g) {
+                                                               int64_t total, const int* bad, TmGeom g) {
+  const bool fill = bad[0] != 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    if (tm_kept(g, i)) continue;
+    if (tm_kept(g, i)) {
+      if (fill) sol[i] = mkc<R>((R)NAN, (R)NAN);
+      continue;
+    }
     cplx<R> u = sol[i];
-    if (u.x == R(0) && u.y == R(0)) continue;
     const double l = L[i];
+    if (u.x == R(0) && u.y == R(0) && isfinite(l) && (!F || isfinite(F[i]))) continue;
     auto rhs = [&](cplx<R> x) { return mkc<R>((R)(l * (double)x.x), (R)(l * (double)x.y)); };
     auto sub = [&](cplx<R> k, double hh) {
       return mkc<R>((R)((double)u.x + hh * (double)k.x), (R)((double)u.y + hh * (double)k.y));
@@ -305,9 +346,12 @@ static int tm_calcN(const ffhip_op* op, const TmGeom& g, void* N, const void* so
   TmArgs a{};
   a.x = sol;
   a.out = N;
+  a.bad = reinterpret_cast<int*>(op->flags);
+  hipLaunchKernelGGL(k_tracer_clear, dim3(1), dim3(1), 0, st, a.bad);
+  FF_LAUNCHED("k_tracer_clear");
   FF_TRY((tm_launch<R, 0>(g, a, st)));
   hipLaunchKernelGGL((k_tracer_outside_zero<R>), dim3(blocks_for(op->spec_count, kTmThreads, 16384)),
-                     dim3(kTmThreads), 0, st, reinterpret_cast<cplx<R>*>(N), op->spec_count, g);
+                     dim3(kTmThreads), 0, st, reinterpret_cast<cplx<R>*>(N), op->spec_count, a.bad, g);
   FF_LAUNCHED("k_tracer_outside_zero");
   return FFHIP_OK;
 }
@@ -327,10 +371,12 @@ static int tm_rk4(ffhip_op* op, const TmGeom& g, const ffhip_rk4* ts, void* sol,
   a.L = reinterpret_cast<const double*>(ts->L);
   a.F = reinterpret_cast<const double*>(ts->filter);
   a.h6 = dt / 6;
+  a.bad = reinterpret_cast<int*>(op->flags);
   for (int64_t k = 0; k < nsteps; ++k) {
     a.x = sol;
     a.out = s1;
     a.h = h2;
+    a.first = k == 0;
     FF_TRY((tm_launch<R, 1>(g, a, st)));
     a.x = s1;
     a.out = s2;
@@ -344,7 +390,7 @@ static int tm_rk4(ffhip_op* op, const TmGeom& g, const ffhip_rk4* ts, void* sol,
     FF_TRY((tm_launch<R, 4>(g, a, st)));
   }
   hipLaunchKernelGGL((k_tracer_outside<R>), dim3(blocks_for(op->spec_count, kTmThreads, 16384)), dim3(kTmThreads), 0,
-                     st, reinterpret_cast<cplx<R>*>(sol), a.L, a.F, h2, dt, a.h6, nsteps, op->spec_count, g);
+                     st, reinterpret_cast<cplx<R>*>(sol), a.L, a.F, h2, dt, a.h6, nsteps, op->spec_count, a.bad, g);
   FF_LAUNCHED("k_tracer_outside");
   return FFHIP_OK;
 }
