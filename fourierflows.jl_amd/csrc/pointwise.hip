@@ -826,6 +826,8 @@ int ffhip_rk4_create(ffhip_rk4** out, const double* Lre, const double* Lim, int 
   t->count = prod(dims, ndim);
   t->prec = prec;
   t->cplx_coef = Lim != nullptr;
+  for (int64_t i = 0; i < t->count; ++i)
+    if (!std::isfinite(Lre[i]) || (Lim && !std::isfinite(Lim[i]))) t->L_finite = false;
   int rc = upload_coef(&t->L, Lre, Lim, t->count);
   if (rc != FFHIP_OK) {
     rk4_free(t);

@@ -34,6 +34,7 @@ struct ffhip_rk4 {
   int prec = FFHIP_F64;
   int cplx_coef = 0;
   void* L = nullptr;  // FP64 real or complex
+  bool L_finite = true;  // no infinity or NaN in L: a zero mode with N = 0 stays zero
   void* scratch[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // sol1, RHS1..RHS4
   void* filter = nullptr;  // Filtered* explicit steppers: FP64 real spectral filter, or null
 };

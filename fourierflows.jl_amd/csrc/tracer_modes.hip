@@ -249,11 +249,12 @@ __global__ void __launch_bounds__(kTmThreads) k_tracer_outside_zero(cplx<R>* N, 
 }
 
 // The same after a run: outside the band the RK4 steps of du/dt = L u, with the
-// stages' roundings (a zero stays one where L and the filter are finite)
+// stages' roundings (zeros stay: all of them where L is finite)
 template <typename R>
 __global__ void __launch_bounds__(kTmThreads) k_tracer_outside(cplx<R>* sol, const double* L, const double* F,
                                                                double h2, double h, double h6, int64_t nsteps,
-                                                               int64_t total, const int* bad, TmGeom g) {
+                                                               int64_t total, bool zeros_stay, const int* bad,
+                                                               TmGeom g) {
   const bool fill = bad[0] != 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
     if (tm_kept(g, i)) {
@@ -261,8 +262,8 @@ __global__ void __launch_bounds__(kTmThreads) k_tracer_outside(cplx<R>* sol, con
       continue;
     }
     cplx<R> u = sol[i];
+    if (zeros_stay && u.x == R(0) && u.y == R(0)) continue;
     const double l = L[i];
-    if (u.x == R(0) && u.y == R(0) && isfinite(l) && (!F || isfinite(F[i]))) continue;
     auto rhs = [&](cplx<R> x) { return mkc<R>((R)(l * (double)x.x), (R)(l * (double)x.y)); };
     auto sub = [&](cplx<R> k, double hh) {
       return mkc<R>((R)((double)u.x + hh * (double)k.x), (R)((double)u.y + hh * (double)k.y));
@@ -390,7 +391,8 @@ static int tm_rk4(ffhip_op* op, const TmGeom& g, const ffhip_rk4* ts, void* sol,
     FF_TRY((tm_launch<R, 4>(g, a, st)));
   }
   hipLaunchKernelGGL((k_tracer_outside<R>), dim3(blocks_for(op->spec_count, kTmThreads, 16384)), dim3(kTmThreads), 0,
-                     st, reinterpret_cast<cplx<R>*>(sol), a.L, a.F, h2, dt, a.h6, nsteps, op->spec_count, a.bad, g);
+                     st, reinterpret_cast<cplx<R>*>(sol), a.L, a.F, h2, dt, a.h6, nsteps, op->spec_count, ts->L_finite,
+                     a.bad, g);
   FF_LAUNCHED("k_tracer_outside");
   return FFHIP_OK;
 }

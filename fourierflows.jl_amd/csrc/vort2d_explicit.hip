@@ -39,12 +39,13 @@ __global__ void k_ximport(const cplx<R>* __restrict__ sol, cplx<R>* __restrict__
 }
 
 // Scatter the kept band back; outside it N is zero and each mode takes its
-// nsteps steps here, rounding where the plan-based path's arrays do.
+// nsteps steps here, rounding where the plan-based path's arrays do (zeros
+// stay: all of them where L is finite).
 template <typename R>
 __global__ void k_xexport(cplx<R>* __restrict__ sol, const cplx<R>* __restrict__ U, const double* __restrict__ L,
                           const double* __restrict__ F, cplx<R>* __restrict__ m1, const cplx<R>* __restrict__ R1,
                           cplx<R>* __restrict__ m2, const cplx<R>* __restrict__ R2, int kind, double h, double h2,
-                          int64_t nsteps, int64_t step0, VortGeom g) {
+                          int64_t nsteps, int64_t step0, bool zeros_stay, VortGeom g) {
   const int64_t total = (int64_t)g.ny * g.nkr;
   const cplx<R> zero = mkc<R>(0, 0);
   const bool f32 = sizeof(R) == 4;
@@ -64,7 +65,7 @@ __global__ void k_xexport(cplx<R>* __restrict__ sol, const cplx<R>* __restrict__
     cplx<R> u = sol[idx];
     cplx<R> r1 = m1 ? m1[idx] : zero, r2 = m1 ? m2[idx] : zero;
     const double l = L[idx];
-    if (u.x != R(0) || u.y != R(0) || r1.x != R(0) || r1.y != R(0) || r2.x != R(0) || r2.y != R(0)) {
+    if (!zeros_stay || u.x != R(0) || u.y != R(0) || r1.x != R(0) || r1.y != R(0) || r2.x != R(0) || r2.y != R(0)) {
       const double f = F ? F[idx] : 1.0;
       for (int64_t k = 0; k < nsteps; ++k) {
         if (kind == 0) {
@@ -197,7 +198,8 @@ static int xrun(ffhip_op* op, VortState* s, ffhip_rk4* ts, int kind, void* sol, 
   hipLaunchKernelGGL((k_xexport<R>), dim3(blocks_for(total, 256, 4096)), dim3(256), 0, st,
                      reinterpret_cast<cplx<R>*>(sol), reinterpret_cast<const cplx<R>*>(s->U),
                      reinterpret_cast<const double*>(ts->L), F, m1p, reinterpret_cast<const cplx<R>*>(ca.N1), m2p,
-                     reinterpret_cast<const cplx<R>*>(ca.N2), kind, dt, h2, nsteps, step0, g);
+                     reinterpret_cast<const cplx<R>*>(ca.N2), kind, dt, h2, nsteps, step0,
+                     ts->L_finite, g);
   FF_LAUNCHED("k_xexport");
   return FFHIP_OK;
 }
