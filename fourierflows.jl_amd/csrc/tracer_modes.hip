@@ -18,9 +18,9 @@
 //
 // An RK4 stage is one kernel over the kept band: it reads the stage state with
 // its neighbours (from cache), the state and L, and writes RHS and the next
-// stage state, so memory bounds it: 256^3 FP32 (2.5 M kept modes) moves about
-// 100 MB in 27 us, 3.8 TB/s (192^3 FP64: 18 us).  With transforms a stage was
-// four kernels and 228 us.
+// stage state, so memory bounds it: 256^3 FP32 (2.5 M kept modes) moves 80 to
+// 140 MB in 20 to 27 us, 4 to 5 TB/s (192^3 FP64: 13 to 19 us).  With
+// transforms a stage was four kernels and 228 us.
 // FP64 stage arithmetic and the state type at every store as in pointwise.hip.
 #include <cmath>
 #include <cstdlib>
@@ -42,8 +42,8 @@ struct TmGeom {
   int tfast, tslow;        // workgroups of a group of planes
   int per_xcd, nblk;
   float inv_fast, inv_slow;
-  double A, B, C, dk, dl, dm;
-  double p[3][2];          // exp(i x0)
+  double dk, dl, dm;
+  double p[3][2];          // (B, C, A) / 2 exp(i x0)
 };
 
 struct TmArgs {
@@ -83,28 +83,28 @@ struct TmField {
   }
 };
 
-// (a, b) = (p z_{k-q}, conj(p) z_{k+q}): *c = their half sum (cos), *s = their difference over 2i (sin)
+// (a, b) = (p z_{k-q}, conj(p) z_{k+q}), p = A / 2 exp(i x0): *c = a + b = (A cos x c)^_k, *s = (a - b) / i =
+// (A sin x c)^_k.  In FP64 for either state type: the velocity's coefficients are FP64 as the grid's are, N is
+// rounded once, which costs FP32 little beside the memory (256^3: 102.4 -> 103.5 us a step; error of N 6.7e-8 -> 2.5e-8).
 template <typename R>
-__device__ __forceinline__ void tm_pair(const double* p, cplx<R> zm, cplx<R> zp, cplx<R>* c, cplx<R>* s) {
-  const R pr = (R)p[0], pi = (R)p[1];
-  const cplx<R> a = mkc<R>(pr * zm.x - pi * zm.y, pr * zm.y + pi * zm.x);
-  const cplx<R> b = mkc<R>(pr * zp.x + pi * zp.y, pr * zp.y - pi * zp.x);
-  *c = mkc<R>(R(0.5) * (a.x + b.x), R(0.5) * (a.y + b.y));
-  *s = mkc<R>(R(0.5) * (a.y - b.y), R(-0.5) * (a.x - b.x));
+__device__ __forceinline__ void tm_pair(const double* p, cplx<R> zm, cplx<R> zp, double2* c, double2* s) {
+  const double ax = p[0] * (double)zm.x - p[1] * (double)zm.y, ay = p[0] * (double)zm.y + p[1] * (double)zm.x;
+  const double bx = p[0] * (double)zp.x + p[1] * (double)zp.y, by = p[0] * (double)zp.y - p[1] * (double)zp.x;
+  *c = make_double2(ax + bx, ay + by);
+  *s = make_double2(ay - by, bx - ax);
 }
 
 template <typename R, bool SLOW>
 __device__ __forceinline__ cplx<R> tm_N(const TmGeom& g, const TmField<R>& f, int kx, int l, int m) {
   auto get = [&](int a, int b, int c) { return SLOW ? f.get_any(g, a, b, c) : f.get(g, a, b, c); };
-  cplx<R> cx, sx, cy, sy, cz, sz;
+  double2 cx, sx, cy, sy, cz, sz;
   tm_pair<R>(g.p[0], get(kx - g.q[0], l, m), get(kx + g.q[0], l, m), &cx, &sx);
   tm_pair<R>(g.p[1], get(kx, l - g.q[1], m), get(kx, l + g.q[1], m), &cy, &sy);
   tm_pair<R>(g.p[2], get(kx, l, m - g.q[2]), get(kx, l, m + g.q[2]), &cz, &sz);
-  const R A = (R)g.A, B = (R)g.B, C = (R)g.C;
-  const R k = (R)(g.dk * (double)kx), ll = (R)(g.dl * (double)l), mm = (R)(g.dm * (double)m);
-  const R sr = k * (A * sz.x + C * cy.x) + ll * (B * sx.x + A * cz.x) + mm * (C * sy.x + B * cx.x);
-  const R si = k * (A * sz.y + C * cy.y) + ll * (B * sx.y + A * cz.y) + mm * (C * sy.y + B * cx.y);
-  return mkc<R>(si, -sr);  // -i (kx U + l V + m W)
+  const double k = g.dk * (double)kx, ll = g.dl * (double)l, mm = g.dm * (double)m;
+  const double sr = k * (sz.x + cy.x) + ll * (sx.x + cz.x) + mm * (sy.x + cx.x);
+  const double si = k * (sz.y + cy.y) + ll * (sx.y + cz.y) + mm * (sy.y + cx.y);
+  return mkc<R>((R)si, (R)-sr);  // -i (kx U + l V + m W)
 }
 
 // What a mode's update reads, and its update.  STAGE 0: N of x to out (both
@@ -300,8 +300,9 @@ static bool tm_geom(const ffhip_op* op, TmGeom* g) {
     if (2 * (int64_t)kmax[d] + g->q[d] >= op->n[d]) return false;
     const double x0 = op->params[3 + d];
     if (!std::isfinite(x0) || !std::isfinite(op->params[d])) return false;
-    g->p[d][0] = std::cos(x0);
-    g->p[d][1] = std::sin(x0);
+    const double amp = 0.5 * op->params[d == 0 ? 1 : d == 1 ? 2 : 0];  // B along x, C along y, A along z
+    g->p[d][0] = amp * std::cos(x0);
+    g->p[d][1] = amp * std::sin(x0);
   }
   g->nkr = (int)op->nkr;
   g->ny = (int)op->n[1];
@@ -322,9 +323,6 @@ static bool tm_geom(const ffhip_op* op, TmGeom* g) {
   g->inv_slow = 1.0f / (float)g->slow;
   g->nblk = (g->tfast + g->tslow) * ((g->KZ + kTmPlanes - 1) / kTmPlanes);
   g->per_xcd = (g->nblk + 7) / 8;
-  g->A = op->params[0];
-  g->B = op->params[1];
-  g->C = op->params[2];
   g->dk = twopi / op->box[0];
   g->dl = twopi / op->box[1];
   g->dm = twopi / op->box[2];
