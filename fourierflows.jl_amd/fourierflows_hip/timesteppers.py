@@ -174,27 +174,51 @@ class RK4TimeStepper(_Handle):
         _lib.call("ffhip_rk4_update", self._h, ptr(sol), ptr(self.RHS1), ptr(self.RHS2), ptr(self.RHS3),
                   ptr(self.RHS4), float(dt), stream_ptr())
 
-    def _stage(self, sol, RHS, x, dt):
-        """``addlinearterm(RHS, x)`` and ``substepsol(sol1, sol, RHS, dt)`` in one pass."""
-        _lib.call("ffhip_rk4_stage", self._h, ptr(self.sol1), ptr(sol), ptr(RHS), ptr(x), float(dt), stream_ptr())
+    def _overridden(self):
+        """True where a subclass (or the object) brings its own ``addlinearterm``,
+        ``substepsol`` or ``update``: then they are called, instead of the one
+        pass that does the work of the library's own."""
+        cls, own = type(self), vars(self)
+        return any(name in own or getattr(cls, name) is not fn for name, fn in _RK4_PASSES)
+
+    def _filter(self, sol):
+        if hasattr(self, "filter_host"):
+            _lib.call("ffhip_rk4_apply_filter", self._h, ptr(sol), stream_ptr())
+
+    def _stage(self, sol, RHS, x, dt, overridden):
+        """``addlinearterm(RHS, x)`` and ``substepsol(sol1, sol, RHS, dt)``."""
+        if overridden:
+            self.addlinearterm(RHS, x)
+            self.substepsol(self.sol1, sol, RHS, dt)
+        else:
+            _lib.call("ffhip_rk4_stage", self._h, ptr(self.sol1), ptr(sol), ptr(RHS), ptr(x), float(dt), stream_ptr())
 
     def stepforward(self, sol, clock, eqn, vars, params, grid):
         """src/timesteppers.jl:237-274 (and the filter, if there is one, in the last pass)."""
         t, dt = clock.t, clock.dt
+        own = self._overridden()
         eqn.calcN(self.RHS1, sol, t, clock, vars, params, grid)
-        self._stage(sol, self.RHS1, sol, dt / 2)
+        self._stage(sol, self.RHS1, sol, dt / 2, own)
         eqn.calcN(self.RHS2, self.sol1, t + dt / 2, clock, vars, params, grid)
-        self._stage(sol, self.RHS2, self.sol1, dt / 2)
+        self._stage(sol, self.RHS2, self.sol1, dt / 2, own)
         eqn.calcN(self.RHS3, self.sol1, t + dt / 2, clock, vars, params, grid)
-        self._stage(sol, self.RHS3, self.sol1, dt)
+        self._stage(sol, self.RHS3, self.sol1, dt, own)
         eqn.calcN(self.RHS4, self.sol1, t + dt, clock, vars, params, grid)
-        _lib.call("ffhip_rk4_last", self._h, ptr(sol), ptr(self.RHS1), ptr(self.RHS2), ptr(self.RHS3),
-                  ptr(self.RHS4), ptr(self.sol1), float(dt), stream_ptr())
+        if own:
+            self.addlinearterm(self.RHS4, self.sol1)
+            self.update(sol, dt)
+            self._filter(sol)
+        else:
+            _lib.call("ffhip_rk4_last", self._h, ptr(sol), ptr(self.RHS1), ptr(self.RHS2), ptr(self.RHS3),
+                      ptr(self.RHS4), ptr(self.sol1), float(dt), stream_ptr())
         clock.advance(1)
 
     def run_fused(self, op, sol, clock, nsteps):
         _lib.call("ffhip_op_rk4_run", op.handle, self._h, ptr(sol), float(clock.dt), int(nsteps), stream_ptr())
         clock.advance(nsteps)
+
+
+_RK4_PASSES = tuple((name, getattr(RK4TimeStepper, name)) for name in ("addlinearterm", "substepsol", "update"))
 
 
 def _attach_filter(ts, eqn, setter, filterkw):
@@ -236,7 +260,6 @@ class FilteredRK4TimeStepper(RK4TimeStepper):
     def __init__(self, eqn, dt=None, dev=None, **filterkw):
         super().__init__(eqn, dt, dev)
         _attach_filter(self, eqn, "ffhip_rk4_set_filter", filterkw)
-
 
 
 class _ExplicitBase(RK4TimeStepper):
@@ -299,8 +322,15 @@ class AB3TimeStepper(_ExplicitBase):
 
     def stepforward(self, sol, clock, eqn, vars, params, grid):
         eqn.calcN(self.RHS, sol, clock.t, clock, vars, params, grid)
-        _lib.call("ffhip_ab3_step", self._h, ptr(sol), ptr(self.RHS), ptr(self.RHSm1), ptr(self.RHSm2),
-                  float(clock.dt), int(clock.step), stream_ptr())
+        args = (self._h, ptr(sol), ptr(self.RHS), ptr(self.RHSm1), ptr(self.RHSm2), float(clock.dt), int(clock.step),
+                stream_ptr())
+        if self._overridden():
+            self.addlinearterm(self.RHS, sol)
+            _lib.call("ffhip_ab3_update", *args)
+            self.RHSm2.copy_(self.RHSm1)
+            self.RHSm1.copy_(self.RHS)
+        else:
+            _lib.call("ffhip_ab3_step", *args)
         clock.advance(1)
 
     def _history(self):
@@ -334,10 +364,17 @@ class LSRK54TimeStepper(_ExplicitBase):
 
     def stepforward(self, sol, clock, eqn, vars, params, grid):
         t, dt = clock.t, clock.dt
+        own = self._overridden()
         for i in range(5):
             eqn.calcN(self.RHS, sol, t + self.C[i] * dt, clock, vars, params, grid)
-            _lib.call("ffhip_lsrk54_full", self._h, ptr(sol), ptr(self.S2), ptr(self.RHS), self.A[i], self.B[i],
-                      float(dt), 1 if i == 4 else 0, stream_ptr())
+            args = (self._h, ptr(sol), ptr(self.S2), ptr(self.RHS), self.A[i], self.B[i], float(dt))
+            if own:
+                self.addlinearterm(self.RHS, sol)
+                _lib.call("ffhip_lsrk54_stage", *args, stream_ptr())
+            else:
+                _lib.call("ffhip_lsrk54_full", *args, 1 if i == 4 else 0, stream_ptr())
+        if own:
+            self._filter(sol)
         clock.advance(1)
 
 
