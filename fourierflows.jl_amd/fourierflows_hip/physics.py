@@ -23,7 +23,7 @@ import types
 import numpy as np
 
 from . import _lib
-from .core import HIP, _tdtype, device_array, prec_of, ptr, stream_ptr, zeros
+from .core import HIP, device_array, prec_of, ptr, stream_ptr, zeros
 from .domains import OneDGrid, Plan, ThreeDGrid, TwoDGrid, ldiv, mul
 from .timesteppers import Equation, Problem
 
@@ -180,17 +180,18 @@ class Diffusion:
         grid's own type and shape that record no derivatives, on lines that fit
         one workgroup; False: nothing was done."""
         torch = __import__("torch")
-        if torch.autograd.forward_ad._current_level >= 0:
-            return False
         plan = grid.rfftplan
         if type(plan) is not Plan or plan.kind != "rfft" or plan.ns != (grid.nx,) or plan.batch != 1:
             return False
-        real, cplx = _tdtype(plan.T), _tdtype(np.result_type(plan.T, np.complex64))
+        f32 = plan.prec == _lib.F32
+        real, cplx = (torch.float32, torch.complex64) if f32 else (torch.float64, torch.complex128)
         forms = ((sol, cplx, grid.nkr), (grid.kr, real, grid.nkr), (params.kappa, real, grid.nx),
                  (vars.cx, real, grid.nx), (vars.cxh, cplx, grid.nkr), (N, cplx, grid.nkr))
+        tangent = torch.autograd.forward_ad.unpack_dual
         for x, dtype, n in forms:
             if type(x) is not torch.Tensor or x.dtype != dtype or x.shape != (n,) or not x.is_contiguous() \
-                    or not x.is_cuda or x.device != sol.device or x.requires_grad or x.is_conj() or x.is_neg():
+                    or not x.is_cuda or x.device != sol.device or x.requires_grad or x.is_conj() or x.is_neg() \
+                    or tangent(x)[1] is not None:
                 return False
         ptrs = [x.data_ptr() for x, _, _ in forms]
         ends = sorted((p, p + x.numel() * x.element_size()) for p, (x, _, _) in zip(ptrs, forms))
@@ -199,6 +200,8 @@ class Diffusion:
         done = C.c_int(0)
         _lib.call("ffhip_diffusion1d_calcN", plan.handle, *ptrs, C.byref(done),
                   stream_ptr())
+        if done.value:  # written in place, as autograd's saved tensors have to know
+            torch.autograd.graph.increment_version((vars.cx, vars.cxh, N))
         return bool(done.value)
 
     @staticmethod
