@@ -227,8 +227,8 @@ __global__ void __launch_bounds__(kMixThreads) k_mrows_c2r(const cplx<R>* __rest
 // c2c along a strided axis: transform (slab, column c) has element i at
 // slab * slab_dist + c + i * stride; a workgroup takes G * ng adjacent columns
 // (in and out may be the same array: a workgroup reads its columns before it
-// writes them).  Each XCD takes a contiguous range of workgroups, so that the
-// lines two of them share stay in one L2.
+// writes them).  Each XCD takes a contiguous range of per_xcd workgroups, so
+// that the lines two of them share stay in one L2; per_xcd = 0: in order.
 template <int DIR, typename R, bool PRIME>
 __global__ void __launch_bounds__(kMixThreads) k_mcols(const cplx<R>* in, cplx<R>* out, MixDev f, int64_t ncols,
                                                       uint32_t stride, int64_t slab_dist, MixShape sh, R scale,
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(kMixThreads) k_mcols(const cplx<R>* in, cplx<R
   __shared__ int table[kMixTable / 4];
   mix_table(f, table, threadIdx.x);
   const MixTile<R> T{reinterpret_cast<cplx<R>*>(msm), sh.G, f.n};
-  const int64_t blk = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  const int64_t blk = per_xcd ? (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8 : blockIdx.x;
   const int64_t col0 = blk * sh.G * sh.ng;
   if (col0 >= ncols) return;  // whole workgroup, before any barrier
   const int left = (int)(ncols - col0 < sh.G * sh.ng ? ncols - col0 : sh.G * sh.ng);
@@ -265,7 +265,7 @@ static MixShape shape(const MixFft& f, int prec, int64_t count, int64_t total, i
   while (s.G * 2 <= gmax && s.G < count && mix_threads(f, 2 * s.G) > 0 && mix_lds(f, 2 * s.G, prec) <= kMixLds / 2 &&
          (s.G < gmin || total >= 2 * s.G * kWgs))
     s.G *= 2;
-  while ((int64_t)s.G * (s.ng + 1) * f.n <= kElems &&
+  while ((int64_t)s.G * s.ng < count && (int64_t)s.G * (s.ng + 1) * f.n <= kElems &&
          (total >= (int64_t)s.G * (s.ng + 1) * kWgs || (gmax == 1 && (int64_t)(s.ng + 1) * f.n <= kRow)) &&
          mix_threads(f, s.G * (s.ng + 1)) > 0)
     ++s.ng;
@@ -343,9 +343,16 @@ static int cols_t(const void* in, void* out, int64_t ncols, int64_t stride, int6
   auto kern = mix_prime_pass(ax.mix) ? k_mcols<DIR, R, true> : k_mcols<DIR, R, false>;
   static bool attr[2] = {false, false};
   FF_TRY(mix_lds_attr(kern, &attr[mix_prime_pass(ax.mix)]));
-  const int64_t per_xcd = ((ncols + B - 1) / B + 7) / 8;
+  // Slabs of fewer than eight workgroups go in order: as ranges, the first of
+  // each slab would all run on the first XCD (block b runs on XCD b % 8) and
+  // the rest of the eight would be empty.  16 x 16 x 2048 mul!, one workgroup a
+  // slab (and no wider than the slab, see shape()): FP32 complex 40 -> 21 us,
+  // 4096 fields of 16 x 16 FP64 complex 68 -> 22 us.
+  const int64_t wgs = (ncols + B - 1) / B;
+  const int64_t per_xcd = nslabs > 1 && wgs < 8 ? 0 : (wgs + 7) / 8;
+  const int64_t gx = per_xcd ? 8 * per_xcd : wgs;
   prof_launch("fft_cols_c2c", 2.0 * ncols * nslabs * ax.n * sizeof(cplx<R>), kern,
-              dim3((unsigned)(8 * per_xcd), (unsigned)nslabs), dim3(mix_wg_threads(ax.mix, B, 8 * per_xcd * nslabs)), mix_lds(ax.mix, B, prec),
+              dim3((unsigned)gx, (unsigned)nslabs), dim3(mix_wg_threads(ax.mix, B, gx * nslabs)), mix_lds(ax.mix, B, prec),
               st, reinterpret_cast<const cplx<R>*>(in), reinterpret_cast<cplx<R>*>(out), mix_dev(ax.mix, ax.mixtw), ncols, (uint32_t)stride, slab_dist, s, (R)scale, (int)per_xcd);
   FF_LAUNCHED("k_mcols");
   return FFHIP_OK;
