@@ -138,7 +138,7 @@ constexpr int fcol_sub() {  // workgroups whose column segments share one 128 B 
 // the next group.  The ranges of a 2D array differ by one group at most: 1025
 // FP32 columns in ranges of nine groups gave seven XCDs 36 workgroups for their
 // 32 compute units and the last one five (2048^2 FP32 mul! + ldiv! 57.7 us,
-// 53.8 us with this split and the loads below).  With many slabs the ranges
+// 53.0 us with this split and the loads below).  With many slabs the ranges
 // are all of the same length gpx, which fills the chip as well.
 __device__ __forceinline__ bool fxcd_split(int b, int nsub, int groups, int gpx, int* group, int* sub) {
   const int x = b % 8;
@@ -171,14 +171,19 @@ __global__ void __launch_bounds__((fcol_cols<R, N>() * (N / fcol_pts(N)))) k_fco
   const int64_t col = col0 + c;
   const bool live = col < ncols;
   const int64_t base = (int64_t)blockIdx.y * slab_dist + (live ? col : 0);
-  // The data before the twiddles, which the first butterflies do not need, and
-  // without a branch (a lane beyond the columns reads column 0 and drops it), so
-  // that every load is in flight before the first wait.
-  cplx<R> v[P];
-#pragma unroll
-  for (int p = 0; p < P; ++p) v[p] = in[base + (int64_t)(tid + p * T) * stride];
+  // The data before the twiddles, which the first butterflies do not need: FP32
+  // 2048 points 7% faster than the other way round, FP64 1024 and 2048 5 and 8%.
+  // FP64 columns of 64 points, whose passes are short, lose 7% so (128 x 64 x
+  // 256 36.5 -> 38.6 us) and ask for the twiddles first.  A lane beyond the
+  // columns keeps its branch: without it the loads took registers (FP64 512
+  // points 95 instead of 68) and up to 4% more time.
+  constexpr bool roots_first = sizeof(R) == 8 && N == 64;
   TwRegs<N, P, R> twr;
-  twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
+  cplx<R> v[P];
+  if constexpr (roots_first) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
+#pragma unroll
+  for (int p = 0; p < P; ++p) v[p] = live ? in[base + (int64_t)(tid + p * T) * stride] : mkc<R>(0, 0);
+  if constexpr (!roots_first) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
   team_fft<N, P, DIR, R>(v, reinterpret_cast<cplx<R>*>(fsm) + c * SL, tid, nullptr, twr);
   if (live) {
 #pragma unroll
