@@ -95,14 +95,19 @@ static int launch_colt(const VortGeom& g, const VortColArgs& a, hipStream_t st) 
   return FFHIP_OK;
 }
 
-// Three teams per column (vort2d_team3.h) up to 256 points and, while the
-// columns fit the chip at once, at 512 and 1024; the single-team kernel beyond.
+// Three teams per column (vort2d_team3.h) up to 256 points and, up to a number
+// of columns, at 512 and 1024; the single-team kernel beyond.
 // Stage 2 on an n x n grid, single team -> three teams, MI355X: FP64 64^2 7.6
 // -> 3.5 us, 128^2 9.0 -> 4.2, 256^2 17.1 -> 5.1, 512^2 17.2 -> 7.4; FP32 64^2
 // 6.2 -> 3.5, 128^2 7.0 -> 4.1, 256^2 12.0 -> 4.7, 512^2 7.8 -> 6.2, 1024^2
 // 14.8 -> 12.5.  With 683 columns (nx = 2048) FP32 loses at 512 (9.5 -> 9.7)
 // and 1024 (19.0 -> 22.7), FP64 at 1024 already with 341 (stage 4: 25.6 ->
-// 32 us, its operands spill).  With many short columns two per workgroup use
+// 32 us, its operands spill).  FP64 512 points, single team -> three teams:
+// stage 1 with 171 tiles of columns (nx = 2048) 21.9 -> 16.0, 257 24.9 -> 23.0,
+// 342 (nx = 4096) 27.1 -> 27.1 and stage 2 28.6 -> 25.4; stage 4, the one with
+// most operands, 171 22.3 -> 19.4, 235 23.7 -> 23.3, 257 25.0 -> 26.5, 342 27.1
+// -> 31.3.  Up to 256 points three teams win at every width up to 4096 (FP64
+// 256 x 4096 23.2 -> 12.3).  With many short columns two per workgroup use
 // the lines better (128-point FP32, nx = 4096: 7.0 -> 5.9 us).
 template <typename R, int N, int STAGE>
 static int launch_col(const VortGeom& g, const VortColArgs& a, hipStream_t st) {
@@ -112,7 +117,8 @@ static int launch_col(const VortGeom& g, const VortColArgs& a, hipStream_t st) {
   } else if constexpr (N == 256) {
     return g.TX <= 96 ? launch_colt<R, N, STAGE, 4, 1>(g, a, st) : launch_colt<R, N, STAGE, 8, 2>(g, a, st);
   } else if constexpr (N == 512 && !f32) {
-    return launch_colt<R, N, STAGE, 8, 1>(g, a, st);
+    if (g.TX <= (STAGE == 4 ? 240 : 344)) return launch_colt<R, N, STAGE, 8, 1>(g, a, st);
+    return launch_col_team<R, N, STAGE>(g, a, st);
   } else {
     if constexpr (N == 512) {
       if (g.TX <= 88) return launch_colt<R, N, STAGE, 8, 1>(g, a, st);
