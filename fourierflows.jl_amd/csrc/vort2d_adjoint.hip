@@ -589,33 +589,13 @@ __global__ void __launch_bounds__(3 * (N / P)) k_varowt(VortGeom g, VortAdjRowAr
 // 9.9 -> 6.8; rows FP64 256^2 9.5 -> 5.0, 512^2 16.1 -> 7.9, FP32 256^2 8.6 ->
 // 4.5, 512^2 7.3 -> 6.3.  Gradient over 20 steps, 4 checkpoints: 512^2 FP64 5.68
 // -> 3.71 ms, 256^2 FP32 3.27 -> 2.24 ms, 512^2 FP32 3.26 -> 2.96 ms.
-template <typename R, int N>
-static bool acol_teams(const VortGeom& g) {
-  return N <= 256 || (N == 512 && (sizeof(R) == 8 || g.TX <= 88));
-}
-
-template <typename R, int N, int STAGE>
-static int launch_acol(const VortGeom& g, const VortAdjColArgs& a, hipStream_t st) {
-  constexpr int P = vcol_pts<R, N>();
-  constexpr size_t sl = team_slice(TeamSched<N, P>::LDS, sizeof(cplx<R>), kCBK);
-  size_t sh = ((acol_pair<R, N>() ? 2 : 1) * kCBK * sl + tw_slots<N, P>()) * sizeof(cplx<R>);
-  auto kern = k_vacol<R, N, P, STAGE>;
-  int per = kCSUB, threads = kCBK * (N / P);
-  const bool teams = acol_teams<R, N>(g);
-  if constexpr (N <= 512) {
-    if (teams) {
-      constexpr int PT = N <= 256 ? 4 : 8;
-      kern = k_vacolt<R, N, PT, STAGE>;
-      sh = 3 * (size_t)TeamSched<N, PT>::LDS * sizeof(cplx<R>);
-      per = kVCB;
-      threads = 3 * (N / PT);
-    }
-  }
-  static bool attr_set[2] = {false, false};
-  if (!attr_set[teams]) {
+template <typename R, int STAGE, typename K>
+static int start_acol(K kern, bool* attr_set, int wgs, int threads, size_t sh, const VortGeom& g,
+                      const VortAdjColArgs& a, hipStream_t st) {
+  if (!*attr_set) {
     FF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)sh));
-    attr_set[teams] = true;
+    *attr_set = true;
   }
   static const char* names[5] = {"vort_adj_col_stage0", "vort_adj_col_stage1", "vort_adj_col_stage2",
                                  "vort_adj_col_stage3", "vort_adj_col_stage4"};
@@ -626,37 +606,78 @@ static int launch_acol(const VortGeom& g, const VortAdjColArgs& a, hipStream_t s
                                           : STAGE == 2 ? 3 * cs + 2 * ds : STAGE == 3 ? 5 * cs + 2 * ds
                                           : (a.cont ? 4 * cs + 4 * ds : 2 * cs));
   const int groups = (g.TX + kXCD - 1) / kXCD * kXCD;
-  prof_launch(names[STAGE], bytes, kern, dim3(groups * per), dim3(threads), sh, st, g, a);
-  FF_LAUNCHED("k_vacol");
+  prof_launch(names[STAGE], bytes, kern, dim3(groups * wgs), dim3(threads), sh, st, g, a);
+  FF_LAUNCHED("k_vacol / k_vacolt");
+  return FFHIP_OK;
+}
+
+template <typename R, int N, int STAGE>
+static int launch_acol_team(const VortGeom& g, const VortAdjColArgs& a, hipStream_t st) {
+  constexpr int P = vcol_pts<R, N>();
+  constexpr size_t sl = team_slice(TeamSched<N, P>::LDS, sizeof(cplx<R>), kCBK);
+  constexpr size_t sh = ((acol_pair<R, N>() ? 2 : 1) * kCBK * sl + tw_slots<N, P>()) * sizeof(cplx<R>);
+  static bool attr_set = false;
+  return start_acol<R, STAGE>(k_vacol<R, N, P, STAGE>, &attr_set, kCSUB, kCBK * (N / P), sh, g, a, st);
+}
+
+template <typename R, int N, int STAGE>
+static int launch_acolt(const VortGeom& g, const VortAdjColArgs& a, hipStream_t st) {
+  constexpr int P = N <= 256 ? 4 : 8;
+  constexpr size_t sh = 3 * (size_t)TeamSched<N, P>::LDS * sizeof(cplx<R>);
+  static bool attr_set = false;
+  return start_acol<R, STAGE>(k_vacolt<R, N, P, STAGE>, &attr_set, kVCB, 3 * (N / P), sh, g, a, st);
+}
+
+template <typename R, int N, int STAGE>
+static int launch_acol(const VortGeom& g, const VortAdjColArgs& a, hipStream_t st) {
+  if constexpr (N <= 256 || (N == 512 && sizeof(R) == 8)) {
+    return launch_acolt<R, N, STAGE>(g, a, st);
+  } else {
+    if constexpr (N == 512) {
+      if (g.TX <= 88) return launch_acolt<R, N, STAGE>(g, a, st);
+    }
+    return launch_acol_team<R, N, STAGE>(g, a, st);
+  }
+}
+
+template <typename R, typename K>
+static int start_arow(K kern, bool* attr_set, int wgs, int threads, size_t sh, const VortGeom& g,
+                      const VortAdjRowArgs& a, hipStream_t st) {
+  if (!*attr_set) {
+    FF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)sh));
+    *attr_set = true;
+  }
+  const double bytes = 5.0 * g.KX * g.ny * sizeof(cplx<R>) + (double)vfield_bytes<R>(g);
+  const int groups = (g.ny / 4 + kXCD - 1) / kXCD * kXCD;
+  prof_launch("vort_adj_row", bytes, kern, dim3(groups * wgs), dim3(threads), sh, st, g, a);
+  FF_LAUNCHED("k_varow / k_varowt");
   return FFHIP_OK;
 }
 
 template <typename R, int N>
-static int launch_arow(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t st) {
+static int launch_arow_team(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t st) {
   constexpr int P = vrow_pts<R, N>();
-  size_t sh =
+  constexpr size_t sh =
       ((size_t)kRRK * team_slice(TeamSched<N, P>::LDS, sizeof(cplx<R>), kRRK) + tw_slots<N, P>()) * sizeof(cplx<R>);
-  auto kern = k_varow<R, N, P>;
-  int per = kRSUB, threads = kRRK * (N / P);
-  constexpr bool teams = N <= 512;
-  if constexpr (teams) {
-    constexpr int PT = N <= 256 ? 4 : 8;
-    kern = k_varowt<R, N, PT>;
-    sh = 3 * (size_t)TeamSched<N, PT>::LDS * sizeof(cplx<R>);
-    per = 2;
-    threads = 3 * (N / PT);
-  }
-  static bool attr_set[2] = {false, false};
-  if (!attr_set[teams]) {
-    FF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)sh));
-    attr_set[teams] = true;
-  }
-  const double bytes = 5.0 * g.KX * g.ny * sizeof(cplx<R>) + (double)vfield_bytes<R>(g);
-  const int groups = (g.ny / 4 + kXCD - 1) / kXCD * kXCD;
-  prof_launch("vort_adj_row", bytes, kern, dim3(groups * per), dim3(threads), sh, st, g, a);
-  FF_LAUNCHED("k_varow");
-  return FFHIP_OK;
+  static bool attr_set = false;
+  return start_arow<R>(k_varow<R, N, P>, &attr_set, kRSUB, kRRK * (N / P), sh, g, a, st);
+}
+
+template <typename R, int N>
+static int launch_arowt(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t st) {
+  constexpr int P = N <= 256 ? 4 : 8;
+  constexpr size_t sh = 3 * (size_t)TeamSched<N, P>::LDS * sizeof(cplx<R>);
+  static bool attr_set = false;
+  return start_arow<R>(k_varowt<R, N, P>, &attr_set, 2, 3 * (N / P), sh, g, a, st);
+}
+
+template <typename R, int N>
+static int launch_arow(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t st) {
+  if constexpr (N <= 512)
+    return launch_arowt<R, N>(g, a, st);
+  else
+    return launch_arow_team<R, N>(g, a, st);
 }
 
 template <typename R, int STAGE>
