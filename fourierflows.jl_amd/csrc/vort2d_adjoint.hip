@@ -582,12 +582,15 @@ __global__ void __launch_bounds__(3 * (N / P)) k_varowt(VortGeom g, VortAdjRowAr
 }
 
 // ----------------------------------------------------------------- launchers
-// Three teams up to 512 points (FP32 512 columns: while they fit the chip at
-// once), the single-team kernels beyond.  Per launch on an n x n grid, single
+// Three teams up to 512 points (FP32 512: on up to 88 tiles of columns and 512
+// rows), the single-team kernels beyond.  Per launch on an n x n grid, single
 // team -> three teams, MI355X: column stages FP64 64^2 9.6 -> 4.3 us, 256^2
 // 19.0 -> 5.5, 512^2 23.5 -> 8.3, FP32 128^2 8.5 -> 4.5, 256^2 12.7 -> 5.3, 512^2
 // 9.9 -> 6.8; rows FP64 256^2 9.5 -> 5.0, 512^2 16.1 -> 7.9, FP32 256^2 8.6 ->
-// 4.5, 512^2 7.3 -> 6.3.  Gradient over 20 steps, 4 checkpoints: 512^2 FP64 5.68
+// 4.5, 512^2 7.3 -> 6.3.  FP32 rows of 512 points are more than fit at once
+// from 640 on and as fast by the single team (1024 rows 6.8 and 6.9), then
+// faster (1280 7.5 and 8.1, 2048 8.6 and 9.7); FP64 rows and columns of 512
+// gain at every size (2048 21.2 -> 16.2 and 27.3 -> 15.0).  Gradient over 20 steps, 4 checkpoints: 512^2 FP64 5.68
 // -> 3.71 ms, 256^2 FP32 3.27 -> 2.24 ms, 512^2 FP32 3.26 -> 2.96 ms.
 template <typename R, int STAGE, typename K>
 static int start_acol(K kern, bool* attr_set, int wgs, int threads, size_t sh, const VortGeom& g,
@@ -674,10 +677,14 @@ static int launch_arowt(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t 
 
 template <typename R, int N>
 static int launch_arow(const VortGeom& g, const VortAdjRowArgs& a, hipStream_t st) {
-  if constexpr (N <= 512)
+  if constexpr (N <= 256 || (N == 512 && sizeof(R) == 8)) {
     return launch_arowt<R, N>(g, a, st);
-  else
+  } else {
+    if constexpr (N == 512) {
+      if (g.ny <= 512) return launch_arowt<R, N>(g, a, st);
+    }
     return launch_arow_team<R, N>(g, a, st);
+  }
 }
 
 template <typename R, int STAGE>
