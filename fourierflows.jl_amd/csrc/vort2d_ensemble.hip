@@ -631,7 +631,10 @@ int ffhip_ensemble_create(ffhip_ensemble** out, int prec, int count, const int64
   }
   if (rc == FFHIP_OK) {
     // Untuned: 8 points per thread everywhere (half the serial work of 16), and
-    // workgroups of 128 threads, or 256 for FP32 members of 512 and more.  Step
+    // workgroups of 128 threads, or 256 with FP32 members of 512 and more and FP64
+    // ones of 1024, whose columns share lines then: FP64 with 128 and 256 threads
+    // 1024^2 213 and 168 us, 2 of them 327 and 213, 4 589 and 352, 4 x 512^2 + 2 x
+    // 1024^2 395 and 244 (16 points from 256 up: 199, 242, 374, 321).  Step
     // time on MI355X, 16 points from 256 up -> this rule: 16 FP32 members (8 x
     // 128^2, 6 x 256^2, 2 x 512^2) 130 -> 98 us, FP64 178 -> 123 us; 64 members
     // FP32 177 -> 148 us, FP64 286 -> 257 us, 200 x 128^2 FP64 247 -> 195 us.
@@ -647,10 +650,9 @@ int ffhip_ensemble_create(ffhip_ensemble** out, int prec, int count, const int64
     if (most <= kEnsTeamMax && ens_points(e) <= (most == 64 ? 1 << 17 : 1 << 18)) {
       v.team = true;
       v.bd = kEnsTeamBd;
-    } else if (prec == FFHIP_F32 && most >= 512) {
+    } else if (most >= (prec == FFHIP_F32 ? 512 : 1024)) {
       v.bd = 256;
     }
-    if (!variant_ok(e, v)) v.bd = 256;  // members of 1024
     // FFHIP_ENS_VARIANT="bd,tcol,trow[,pair]" (thresholds 128, 256, 512 or 2048; pair 0 or 1)
     // fixes the untuned variant
     if (const char* ev = getenv("FFHIP_ENS_VARIANT")) {
