@@ -43,7 +43,11 @@ int fused_etdrk4_run(ffhip_op* op, ffhip_etdrk4* ts, void* sol, int64_t nsteps, 
 int fused_explicit_run(ffhip_op* op, ffhip_rk4* ts, int kind, void* sol, double dt, int64_t nsteps, int64_t step0,
                        void* m1, void* m2, bool* done, hipStream_t st);
 // LSRK54 coefficients (src/timesteppers.jl:330-345), Carpenter & Kennedy (1994)
-extern const double kLsrkA[5], kLsrkB[5];
+inline constexpr double kLsrkA[5] = {0.0, -567301805773.0 / 1357537059087.0, -2404267990393.0 / 2016746695238.0,
+                                     -3550918686646.0 / 2091501179385.0, -1275806237668.0 / 842570457699.0};
+inline constexpr double kLsrkB[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.0 / 13612068292357.0,
+                                     1720146321549.0 / 2090206949498.0, 3134564353537.0 / 4481467310338.0,
+                                     2277821191437.0 / 14882151754819.0};
 // fused tracer RK4 (tracer3d_fused.hip)
 int tracer_fused_create(ffhip_op* op);
 void tracer_fused_destroy(ffhip_op* op);

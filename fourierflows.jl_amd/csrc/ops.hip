@@ -402,12 +402,6 @@ static int rk4_run_generic(ffhip_op* op, ffhip_rk4* ts, void* sol, double dt, in
   return FFHIP_OK;
 }
 
-const double kLsrkA[5] = {0.0, -567301805773.0 / 1357537059087.0, -2404267990393.0 / 2016746695238.0,
-                                 -3550918686646.0 / 2091501179385.0, -1275806237668.0 / 842570457699.0};
-const double kLsrkB[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.0 / 13612068292357.0,
-                                 1720146321549.0 / 2090206949498.0, 3134564353537.0 / 4481467310338.0,
-                                 2277821191437.0 / 14882151754819.0};
-
 // ForwardEuler (kind 0), AB3 (kind 1) and LSRK54 (kind 2), filtered when ts
 // carries a filter, with a built-in operator (src/timesteppers.jl:112-149,
 // 389-414, 630-666).  step0 = clock.step at entry (AB3 starts with 3 Euler

@@ -81,13 +81,8 @@ __global__ void k_xexport(cplx<R>* __restrict__ sol, const cplx<R>* __restrict__
           cplx<R> s2 = zero;
           for (int i = 0; i < 5; ++i) {
             // the coefficients in the state's type, as the stages on the band take them
-            constexpr double A[5] = {0.0, -567301805773.0 / 1357537059087.0, -2404267990393.0 / 2016746695238.0,
-                                     -3550918686646.0 / 2091501179385.0, -1275806237668.0 / 842570457699.0};
-            constexpr double B[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.0 / 13612068292357.0,
-                                     1720146321549.0 / 2090206949498.0, 3134564353537.0 / 4481467310338.0,
-                                     2277821191437.0 / 14882151754819.0};
-            s2 = xlsrk_s2<R>(s2, xrhs<R>(l, u, zero), f32 ? (double)(float)A[i] : A[i], h);
-            u = xadd<R>(u, s2, f32 ? (double)(float)B[i] : B[i]);
+            s2 = xlsrk_s2<R>(s2, xrhs<R>(l, u, zero), f32 ? (double)(float)kLsrkA[i] : kLsrkA[i], h);
+            u = xadd<R>(u, s2, f32 ? (double)(float)kLsrkB[i] : kLsrkB[i]);
           }
         } else {
           const cplx<R> q1 = xrhs<R>(l, u, zero);
