@@ -7,8 +7,8 @@
 // between stages.
 //
 // Measured on MI355X, FilteredRK4 at 512^2 FP32: 206 us per step on the
-// plan-based path, 63 us here (row passes 5.8 us, column stages 8 to 9 us:
-// latency, as in the ETDRK4 steps).
+// plan-based path, 51 us here (row passes 4.8 us, column stages 6.2 us, of which
+// 0.8 and 0.6 are VALU issue: latency, as in the ETDRK4 steps).
 #include "vort2d_col.h"
 
 namespace ffhip {

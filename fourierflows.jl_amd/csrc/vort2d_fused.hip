@@ -176,11 +176,13 @@ static size_t row_lds() {
   return (kRRK * sl + tw_slots<N, vrow_pts<R, N>()>()) * sizeof(cplx<R>);
 }
 
-// Three-team passes (two transforms side by side per column or row pair).
-// Measured on MI355X at 2048^2 with the register-twiddle single-team
-// kernels: slower in FP32 (the single-team kernels keep two waves per SIMD
-// busy) and in FP64 (1953 vs 1891 steps/s with both off), so off by default.
-// FFHIP_COL3 / FFHIP_ROW3: 0 off (default), 1 FP64 only, 2 FP32 and FP64.
+// Three-team passes of 1024- and 2048-point lines (vcol3_body, vrow3_body, with
+// the twiddles in LDS; the shorter lines' are in vort2d_team3.h and do not
+// depend on these switches).  Measured on MI355X at 2048^2 with the
+// register-twiddle single-team kernels: slower in FP32 (the single-team kernels
+// keep two waves per SIMD busy) and in FP64 (1953 steps/s with both off, 1891
+// with both on), so off by default.  FFHIP_COL3 / FFHIP_ROW3: 0 off (default),
+// 1 FP64 only, 2 FP32 and FP64; the explicit steppers' columns stay as they are.
 static bool use3(const char* var, bool f32) {
   const char* e = getenv(var);
   const int mode = e ? atoi(e) : 0;

@@ -53,7 +53,9 @@ class BuiltinOperator:
 
     @property
     def fused(self):
-        """True when libffhip steps this operator's grid with fused kernels."""
+        """True when the operator holds the fused state made with it: the
+        power-of-two vorticity grids (which also run the adjoint) and tracers.
+        Other vorticity grids step fused too, on a state made at the first run."""
         v = C.c_int()
         _lib.call("ffhip_op_is_fused", self._h, C.byref(v))
         return bool(v.value)

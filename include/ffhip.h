@@ -288,7 +288,10 @@ int ffhip_op_checkpoint_id(const ffhip_op* op, int64_t* id);
 int ffhip_op_rk4_adjoint(ffhip_op* op, ffhip_rk4* ts, const void* lamT, void* lam0, double dt, int64_t nsteps,
                          void* stream);
 
-/* Is the fused path active for this operator (power-of-two 2D vorticity grid)? */
+/* Does this operator hold the fused state made with it (power-of-two 2D vorticity
+ * grids, which also run the adjoint, and power-of-two 3D tracers)?  Other
+ * vorticity grids that step fused make their state at the first run, and the
+ * tracer on boxes of multiples of 2 pi steps without one: 0 there. */
 int ffhip_op_is_fused(const ffhip_op* op, int* fused);
 
 /* ---------------------------------------------------------------- ensembles
