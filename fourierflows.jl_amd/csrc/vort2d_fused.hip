@@ -325,8 +325,11 @@ static int launch_rowt(const VortGeom& g, const VortRowArgs& a, hipStream_t st) 
 // between (FP32 512: 4.8 us at 512^2 against 5.1 us by three teams).
 // Row pass on an n x n grid, single team -> three teams, MI355X: FP64 64^2 5.1
 // -> 3.2 us, 128^2 6.2 -> 3.9, 256^2 9.5 -> 4.4, 512^2 9.9 -> 5.9, 1024^2 15.4
-// -> 14.0; FP32 64^2 3.9 -> 3.0, 128^2 4.6 -> 3.6, 256^2 7.0 -> 4.0.  Two
-// pairs per workgroup from 2048 rows of 256 (FP32 6.2 -> 5.9 us).
+// -> 14.0; FP32 64^2 3.9 -> 3.0, 128^2 4.6 -> 3.6, 256^2 7.0 -> 4.0.  On 4096
+// rows three teams win or draw as well (FP64 512 points 28.4 -> 21.4, 1024 48.0
+// -> 45.6, FP32 128 points 6.6 -> 6.6), also where they store the stage fields
+// (2048 rows of 1024 FP64 32.5 -> 28.7).  Two pairs per workgroup from 2048 rows
+// of 256 (FP32 6.2 -> 5.9 us).
 template <typename R, int N>
 static int launch_row(const VortGeom& g, const VortRowArgs& a, hipStream_t st) {
   if constexpr (N <= 128) {
