@@ -396,12 +396,12 @@ static Radices to_radices(const Axis& ax) {
 // FP32 9.9 against 11.2 us and 11.3 against 13.4, FP64 13.8 against 14.1 and
 // 14.8 against 16.3; the same up to 2^15 rows).  r2c is so at 2^16 rows (FP32
 // 7.6 against 8.3), not at 2^18 (12.6 against 11.6).
-static bool row8(const Axis& ax) { return ax.n == 8 && ax.lds; }
+static bool row8(const Axis& ax, int64_t nrows) { return ax.n == 8 && ax.lds && nrows >= (1 << 15); }
 
 template <typename R>
 static int run_rows_c2c(const cplx<R>* in, cplx<R>* out, int64_t nrows, const Axis& ax, int dir, R scale,
                         ffhip_plan* p, hipStream_t st) {
-  if (ax.mixed && !row8(ax)) return mix_rows_c2c(p->prec, in, out, nrows, ax, dir, (double)scale, st);
+  if (ax.mixed && !row8(ax, nrows)) return mix_rows_c2c(p->prec, in, out, nrows, ax, dir, (double)scale, st);
   const int n = (int)ax.n;
   if (ax.lds) {
     int nb = ax.nb;
@@ -453,7 +453,7 @@ template <typename R>
 static int run_rows_r2c(const R* in, cplx<R>* out, int64_t nrows, ffhip_plan* p, hipStream_t st) {
   const Axis& ax = p->ax[0];
   if (ax.fast) return fast_rows_r2c(p->prec, in, out, nrows, ax, p->rtw, st);
-  if (ax.mixed && !(row8(ax) && nrows < (1 << 17))) return mix_rows_r2c(p->prec, in, out, nrows, ax, p->rtw, st);
+  if (ax.mixed && !(row8(ax, nrows) && nrows < (1 << 17))) return mix_rows_r2c(p->prec, in, out, nrows, ax, p->rtw, st);
   const int m = (int)ax.n;
   const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(ax.tw);
   const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p->rtw);
@@ -481,7 +481,7 @@ template <typename R>
 static int run_rows_c2r(const cplx<R>* in, R* out, int64_t nrows, R scale, ffhip_plan* p, hipStream_t st) {
   const Axis& ax = p->ax[0];
   if (ax.fast) return fast_rows_c2r(p->prec, in, out, nrows, ax, p->rtw, (double)scale, st);
-  if (ax.mixed && !row8(ax)) return mix_rows_c2r(p->prec, in, out, nrows, ax, p->rtw, (double)scale, st);
+  if (ax.mixed && !row8(ax, nrows)) return mix_rows_c2r(p->prec, in, out, nrows, ax, p->rtw, (double)scale, st);
   const int m = (int)ax.n;
   const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(ax.tw);
   const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p->rtw);

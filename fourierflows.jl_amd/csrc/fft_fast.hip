@@ -138,7 +138,7 @@ constexpr int fcol_sub() {  // workgroups whose column segments share one 128 B 
 // the next group.  The ranges of a 2D array differ by one group at most: 1025
 // FP32 columns in ranges of nine groups gave seven XCDs 36 workgroups for their
 // 32 compute units and the last one five (2048^2 FP32 mul! + ldiv! 57.7 us,
-// 53.0 us with this split and the loads below).  With many slabs the ranges
+// 53.8 us with this split and the loads below).  With many slabs the ranges
 // are all of the same length gpx, which fills the chip as well.
 __device__ __forceinline__ bool fxcd_split(int b, int nsub, int groups, int gpx, int* group, int* sub) {
   const int x = b % 8;
@@ -153,7 +153,7 @@ __device__ __forceinline__ bool fxcd_split(int b, int nsub, int groups, int gpx,
 // Transform (slab s, column c) has element i at s * slab_dist + c + i * stride;
 // in and out may be the same array (each element is read and written by the
 // same thread, reads first).
-template <typename R, int N, int DIR>
+template <typename R, int N, int DIR, bool ROOTS_FIRST>
 __global__ void __launch_bounds__((fcol_cols<R, N>() * (N / fcol_pts(N)))) k_fcol(
     const cplx<R>* in, cplx<R>* out, const cplx<R>* __restrict__ roots, int64_t ncols, int64_t stride,
     int64_t slab_dist, R scale, int groups, int gpx) {
@@ -171,19 +171,17 @@ __global__ void __launch_bounds__((fcol_cols<R, N>() * (N / fcol_pts(N)))) k_fco
   const int64_t col = col0 + c;
   const bool live = col < ncols;
   const int64_t base = (int64_t)blockIdx.y * slab_dist + (live ? col : 0);
-  // The data before the twiddles, which the first butterflies do not need: FP32
-  // 2048 points 7% faster than the other way round, FP64 1024 and 2048 5 and 8%.
-  // FP64 columns of 64 points, whose passes are short, lose 7% so (128 x 64 x
-  // 256 36.5 -> 38.6 us) and ask for the twiddles first.  A lane beyond the
-  // columns keeps its branch: without it the loads took registers (FP64 512
-  // points 95 instead of 68) and up to 4% more time.
-  constexpr bool roots_first = sizeof(R) == 8 && N == 64;
+  // The data before the twiddles, which the first butterflies do not need (but
+  // see fcol_roots_first).  FP32 lanes beyond the columns read column 0 and drop
+  // it, so that every load is in flight before the first wait; in FP64 that took
+  // registers (512 points 95 instead of 68) and up to 4% more time.
   TwRegs<N, P, R> twr;
   cplx<R> v[P];
-  if constexpr (roots_first) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
+  if constexpr (ROOTS_FIRST) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
 #pragma unroll
-  for (int p = 0; p < P; ++p) v[p] = live ? in[base + (int64_t)(tid + p * T) * stride] : mkc<R>(0, 0);
-  if constexpr (!roots_first) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
+  for (int p = 0; p < P; ++p)
+    v[p] = sizeof(R) == 4 || live ? in[base + (int64_t)(tid + p * T) * stride] : mkc<R>(0, 0);
+  if constexpr (!ROOTS_FIRST) twr_fill_roots<N, P, 1, R, TwRegs<N, P, R>::NR>(twr, roots, tid);
   team_fft<N, P, DIR, R>(v, reinterpret_cast<cplx<R>*>(fsm) + c * SL, tid, nullptr, twr);
   if (live) {
 #pragma unroll
@@ -273,8 +271,19 @@ int fast_rows_c2r(int prec, const void* in, void* out, int64_t nrows, const Axis
                            : rows_c2r_t<double>(in, out, nrows, ax, rtw, scale, st);
 }
 
-template <typename R, int N, int DIR>
-static int cols_n_dir(const void* in, void* out, int64_t ncols, int64_t stride, int64_t nslabs, int64_t slab_dist,
+// Data first gains where a pass is long or the chip has few wavefronts: FP32
+// 2048 points 5%, FP64 1024 and 2048 5 and 8%, FP64 128 points on 17 columns 11.0
+// -> 10.0 us.  On many FP64 columns of up to 512 points, which fill the chip, the
+// twiddles that are asked for last cost more than that hides (data first ->
+// twiddles first: 64 points on 65 x 256 columns 38.5 -> 35.9 us, 256 on 33 x 256
+// 58.2 -> 55.0, 512 on 9 x 256 76.3 -> 69.1, the same within 2% at 2000 columns).
+template <typename R, int N>
+constexpr bool fcol_roots_first() {
+  return sizeof(R) == 8 && N <= 512;
+}
+
+template <typename R, int N, int DIR, bool ROOTS_FIRST>
+static int cols_start(const void* in, void* out, int64_t ncols, int64_t stride, int64_t nslabs, int64_t slab_dist,
                       const Axis& ax, double scale, hipStream_t st) {
   constexpr int P = fcol_pts(N);
   constexpr int C = fcol_cols<R, N>();
@@ -283,7 +292,7 @@ static int cols_n_dir(const void* in, void* out, int64_t ncols, int64_t stride, 
   const size_t sh = (size_t)C * SL * sizeof(cplx<R>);
   static bool attr = false;
   if (!attr) {
-    FF_TRY(set_lds(k_fcol<R, N, DIR>, sh));
+    FF_TRY(set_lds(k_fcol<R, N, DIR, ROOTS_FIRST>, sh));
     attr = true;
   }
   FF_CHECK(nslabs <= 65535, FFHIP_ERR_UNSUPPORTED, "fast column pass: %lld slabs", (long long)nslabs);
@@ -292,12 +301,22 @@ static int cols_n_dir(const void* in, void* out, int64_t ncols, int64_t stride, 
   const int64_t gx = gpx * 8 * SUB;
   FF_CHECK(gx < (1LL << 31), FFHIP_ERR_UNSUPPORTED, "fast column pass: %lld columns", (long long)ncols);
   const double bytes = 2.0 * ncols * nslabs * N * sizeof(cplx<R>);
-  prof_launch("fft_cols_c2c", bytes, k_fcol<R, N, DIR>, dim3((unsigned)gx, (unsigned)nslabs), dim3(C * (N / P)), sh,
-              st, reinterpret_cast<const cplx<R>*>(in), reinterpret_cast<cplx<R>*>(out),
+  prof_launch("fft_cols_c2c", bytes, k_fcol<R, N, DIR, ROOTS_FIRST>, dim3((unsigned)gx, (unsigned)nslabs),
+              dim3(C * (N / P)), sh, st, reinterpret_cast<const cplx<R>*>(in), reinterpret_cast<cplx<R>*>(out),
               reinterpret_cast<const cplx<R>*>(ax.tw), ncols, stride, slab_dist, (R)scale, (int)groups,
               nslabs > 1 ? (int)gpx : 0);
   FF_LAUNCHED("k_fcol");
   return FFHIP_OK;
+}
+
+template <typename R, int N, int DIR>
+static int cols_n_dir(const void* in, void* out, int64_t ncols, int64_t stride, int64_t nslabs, int64_t slab_dist,
+                      const Axis& ax, double scale, hipStream_t st) {
+  if constexpr (fcol_roots_first<R, N>()) {
+    if (ncols * nslabs >= 2048)
+      return cols_start<R, N, DIR, true>(in, out, ncols, stride, nslabs, slab_dist, ax, scale, st);
+  }
+  return cols_start<R, N, DIR, false>(in, out, ncols, stride, nslabs, slab_dist, ax, scale, st);
 }
 
 template <typename R, int N>

@@ -14,7 +14,7 @@ EPS = {np.float32: 2.0**-24, np.float64: 2.0**-53}
 
 @pytest.mark.parametrize("T", [np.float32, np.float64])
 @pytest.mark.parametrize("kind,nx", [("rfft", 16), ("fft", 8)])
-@pytest.mark.parametrize("rows", [1, 63, 1000, (1 << 17) - 1, 1 << 17])
+@pytest.mark.parametrize("rows", [1, 63, 1000, (1 << 15) - 1, 1 << 15, (1 << 17) - 1, 1 << 17])
 def test_rows(rows, kind, nx, T):
     rng = np.random.default_rng(rows)
     x = rng.standard_normal((rows, nx))

@@ -13,12 +13,14 @@ EPS = {np.float32: 2.0**-24, np.float64: 2.0**-53}
 
 
 # slabs of one workgroup and of part of one, of a few, of seven, eight and more,
-# with a batch of fields and as the planes of a 3D field
+# with a batch of fields and as the planes of a 3D field; columns of 64 to 512
+# points on both sides of 2048 in all
 @pytest.mark.parametrize("T", [np.float32, np.float64])
 @pytest.mark.parametrize("kind", ["rfft", "fft"])
 @pytest.mark.parametrize("ns,batch", [((2, 16), 33), ((16, 16), 300), ((12, 20), 65), ((6, 96), 17), ((96, 96), 9),
                                       ((222, 48), 5), ((256, 30), 6), ((500, 12), 3), ((10, 14, 50), 1),
-                                      ((16, 20, 9), 4)])
+                                      ((16, 20, 9), 4), ((62, 64), 65), ((62, 128), 63), ((62, 512), 64),
+                                      ((126, 256), 33)])
 def test_transforms(ns, batch, kind, T):
     rng = np.random.default_rng(batch)
     shape = (batch,) + tuple(reversed(ns))
